@@ -32,6 +32,10 @@ void free_qweight(QWeight& w) {
   if (w.s) (void)hipFree(w.s);
   w.q = nullptr;
   w.s = nullptr;
+  for (WPlanes& p : w.pl) {
+    if (p.owned) (void)hipFree(p.p);
+    p = WPlanes{};
+  }
 }
 
 void upload_qweight(hipStream_t st, const uint8_t* bytes, size_t nbytes, uint32_t type, size_t rows, size_t cols,
@@ -72,6 +76,7 @@ struct hos_ctx {
   DevMem ws, t0, t1, t2, t3, t4, t5;
   DevMem ops[8];  // scratch of the op-level entry points (ops.hip)
   int passes = 1;
+  size_t plane_credit = 0;  // ensure_planes
   hipEvent_t tev[2] = {nullptr, nullptr};  // hos_hip_timer_begin / _end
   bool tarmed = false;                     // a timer_begin not yet closed by a timer_end
   static constexpr size_t kWs = 256ull << 20;
@@ -99,7 +104,7 @@ int guard(hos_ctx* c, F&& f) {
   }
 }
 
-const QWeight& get_qw(hos_ctx* c, uint64_t key) {
+QWeight& get_qw(hos_ctx* c, uint64_t key) {
   auto it = c->qw.find(key);
   HOS_REQUIRE(it != c->qw.end(), HOS_E_INVALID, "no quantized weight uploaded under key " + std::to_string(key));
   return it->second;
@@ -135,13 +140,14 @@ H16 operand_h16(hos_ctx* c, long long K, size_t t) {
 
 void qgemm_dev(hos_ctx* c, bool dx, uint64_t key, const float* in_dev, size_t t, float* out_dev,
                const GemmEpi* lora = nullptr) {
-  const QWeight& w = get_qw(c, key);
+  QWeight& w = get_qw(c, key);
   long long K = dx ? w.rows : w.cols;
   long long N = dx ? w.cols : w.rows;
   HOS_REQUIRE(in_dev && out_dev, HOS_E_INVALID, "qgemm: null pointer");
   H16 a = operand_h16(c, K, t);
   launch_to_h16(in_dev, K, (long long)t, K, a, c->stream);
   c->ws.ensure(hos_ctx::kWs);
+  ensure_planes(w, dx, c->passes, (long long)t, &c->plane_credit, c->stream);
   GemmEpi epi = lora ? *lora : GemmEpi{};
   epi.out = out_dev;
   epi.ldo = N;
@@ -340,8 +346,9 @@ int hos_hip_time_qgemm(hos_ctx* c, int which, uint64_t key, const float* in_dev,
                        float* avg_ms) {
   return guard(c, [&] {
     HOS_REQUIRE(in_dev && out_dev && avg_ms && iters > 0, HOS_E_INVALID, "time_qgemm: bad arguments");
-    const QWeight& w = get_qw(c, key);
+    QWeight& w = get_qw(c, key);
     bool dx = which == 1;
+    ensure_planes(w, dx, c->passes, (long long)t, &c->plane_credit, c->stream);
     long long K = dx ? w.rows : w.cols, N = dx ? w.cols : w.rows;
     H16 a = operand_h16(c, K, t);
     launch_to_h16(in_dev, K, (long long)t, K, a, c->stream);

@@ -68,12 +68,23 @@ inline int ceil_div(long long a, long long b) { return (int)((a + b - 1) / b); }
 //   Q8_0: q = int8 [N][K],     s = f32 d              per (row, 32 cols)
 //   Q4_K: q = u8   [N][K/2]    (col 2i low nibble, 2i+1 high), s = f32 {d·sc, dmin·m} per (row, 32)
 //   Q6_K: q = int8 [N][K],     s = f32 d·sc           per (row, 16 cols)
+// A frozen weight dequantized once into fp16 planes (hi = fp16(w), lo = fp16(w − hi)) in MFMA fragment order, for one
+// GEMM direction (planes.hip): out[m][n] = Σ_c A[m][c]·B(n, c), with n the weight's rows and c its columns (forward)
+// or the other way round (dX). Fragment (nb, ks, plane) is 1 KB: lane l holds column n = 16·nb + (l & 15),
+// c = 32·ks + 8·(l >> 4) .. +7. With experts, each expert's block is laid out on its own, one after the other.
+struct WPlanes {
+  half_t* p = nullptr;
+  int planes = 0;  // 1: hi only, 2: hi and lo
+  bool owned = false;
+};
+
 struct QWeight {
   uint32_t type = 0;
   int64_t rows = 0, cols = 0;
   void* q = nullptr;
   float* s = nullptr;
   size_t q_bytes = 0, s_bytes = 0;
+  WPlanes pl[2];  // forward, dX
 };
 
 // An fp16 GEMM operand with an exact power-of-two scale per row:

@@ -139,6 +139,13 @@ struct GemmEpi {
   // an activation row block), 1 = rows fastest (they share a weight column strip: for outputs many tiles wide,
   // such as the vocabulary head, each strip is then fetched once instead of once per row block).
   int rows_fastest = 0;
+  // The rank-r factors as the plane GEMM reads them (optional beside U and L: it makes them itself otherwise). Uf: bf16
+  // hi plane of U divided by the operand's row scale, 32 columns per segment (or the rank padded to 32), row stride
+  // ldf, the lo plane ulo elements further on; Lf: scale·L as bf16 fragments [column / 16][rank / 32][plane][lane][8],
+  // lane l holding column l & 15, ranks 8·(l >> 4) .. +7. Padding is zero in both.
+  const __bf16* Uf = nullptr;
+  const __bf16* Lf = nullptr;
+  long long ldf = 0, ulo = 0;
   // Deferred reduction (host pointer, may be null): a launch split over the contraction leaves its partials in the
   // workspace, stores the split count here and launches no reduction — the consumer reads the partials (SplitSrc);
   // an unsplit launch writes its output as usual and stores 1.
@@ -176,6 +183,35 @@ void launch_qgemm_fwd(const QWeight& w, H16 a, long long lda, long long M, GemmE
 // dX[M, W.cols] = dY[M, W.rows] · deq(W), dY an fp16 row-scaled operand with row stride lda.
 void launch_qgemm_dx(const QWeight& w, H16 a, long long lda, long long M, GemmEpi epi, float* ws, size_t ws_bytes,
                      int passes, hipStream_t st);
+// ---- planes.hip / plane_gemm.hip ----
+// Planes a launch in this precision mode reads (hi, or hi and lo).
+inline int planes_for(int passes) { return passes >= 3 ? 2 : 1; }
+size_t planes_bytes(const QWeight& w, bool dx, int planes, int groups);
+// Dequantize w into planes at dst (groups: experts stacked in w, each laid out on its own).
+void build_planes(const QWeight& w, bool dx, int planes, int groups, half_t* dst, hipStream_t st);
+// Whether a launch of M rows on this weight takes the plane GEMM once the planes are there (groups > 1: grouped).
+bool plane_gemm_wanted(const QWeight& w, bool dx, int passes, long long M, int groups = 1);
+// Whether planes of this size may be allocated: they never take the card's free memory below half of its total, so
+// a model that fills the card keeps its quantized weights alone.
+bool planes_fit(size_t bytes);
+// Allocate and build the planes a launch wants if they are missing and fit (not while the stream is captured). credit:
+// bytes the caller's context may still allocate before the free memory is looked at again.
+void ensure_planes(QWeight& w, bool dx, int passes, long long M, size_t* credit, hipStream_t st);
+// One fragment column block of a rank-r factor to lay out as GemmEpi::Lf: `rank` rows of `cols` consecutive floats at
+// src + off (row stride ld), block nb, written at dst (all its rank steps).
+struct RankItem {
+  long long off, dst;
+  int ld, rank, cols, nb;
+  float scale;
+};
+// Lay out e.U / e.L as e.Uf / e.Lf at the end of ws (shrinking *ws_bytes); false if they do not fit.
+bool prepare_rank(GemmEpi& e, const float* rinv, long long M, long long N, float* ws, size_t* ws_bytes, hipStream_t st);
+void launch_rank_frags(const RankItem* items, int n, const float* src, __bf16* dst, hipStream_t st);
+// The GEMM on w.pl[dx]; false when this launch is none of its cases (the caller runs the dequantizing kernel).
+bool launch_plane_gemm(bool dx, const QWeight& w, H16 a, long long lda, long long M, GemmEpi epi, float* ws,
+                       size_t ws_bytes, int passes, hipStream_t st);
+bool launch_plane_gemm_grouped(bool dx, const QWeight& w, GroupSched gs, H16 a, long long lda, GemmEpi epi, int passes,
+                               hipStream_t st);
 // f32 [M, K] (row stride ldx) -> fp16 row-scaled operand (row stride K); residual too when out.lo is set.
 void launch_to_h16(const float* x, long long ldx, long long M, long long K, H16 out, hipStream_t st);
 // n samples of N(0, stddev²) from a counter-based hash of (seed, index) (synthetic weights on the device)

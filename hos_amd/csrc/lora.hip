@@ -441,7 +441,16 @@ struct RowsRed {
   float* C;
   long long ldc;
 };
-__global__ void lora_rows_reduce(int gx, int RB, int NC, int M, int n, RowsRed r0, RowsRed r1) {
+// One value of a rows product (column c of n = nt·r) as the plane GEMM's rank factor.
+__device__ __forceinline__ void put_u(const UOut& u, int r, long long row, int c, float v, float rinv) {
+  const float x = v * __uint_as_float((254u << 23) - __float_as_uint(rinv));  // / rinv, a power of two
+  const __bf16 h = (__bf16)x;
+  __bf16* d = u.p + row * u.ld + (c / r) * u.slot + c % r;
+  d[0] = h;
+  d[u.lo] = (__bf16)(x - (float)h);
+}
+__global__ void lora_rows_reduce(int gx, int RB, int NC, int M, int n, RowsRed r0, RowsRed r1, UOut uo = UOut{}, int r = 1,
+                                 const float* rinv = nullptr) {
   const RowsRed& rd = blockIdx.y ? r1 : r0;
   if (rd.S <= 1) return;
   const int E = RB * NC;
@@ -449,7 +458,9 @@ __global__ void lora_rows_reduce(int gx, int RB, int NC, int M, int n, RowsRed r
   if (i >= (long long)gx * E) return;
   const int bx = (int)(i / E), e = (int)(i % E), rr = e / NC, c = e % NC, row = bx * RB + rr;
   if (row >= M || c >= n) return;
-  rd.C[(long long)row * rd.ldc + c] = rd.alpha * sum_parts(rd.part, rd.S, gx, bx, E, e);
+  const float v = rd.alpha * sum_parts(rd.part, rd.S, gx, bx, E, e);
+  rd.C[(long long)row * rd.ldc + c] = v;
+  if (uo.p) put_u(uo, r, row, c, v, rinv[row]);
 }
 // One thread per output element of every block of both jobs (job a's elements first).
 __device__ __forceinline__ void cols_reduce_one(const ColsJobDev& jb, const float* part, int S, long long i) {
@@ -496,7 +507,7 @@ typedef _Float16 h8l __attribute__((ext_vector_type(8)));
 template <int NJ, int RT>
 __global__ void __launch_bounds__(64 * R16_NW) lora_rows16_kernel(int M, int K, int kchunk, float alpha, HIn xh,
                                                                   long long ldx, B16 bt, long long ldb, RowsSeg sg,
-                                                                  float* __restrict__ C, long long ldc, float* part) {
+                                                                  float* __restrict__ C, long long ldc, float* part, UOut uo) {
   constexpr int NC = NJ * 16, E = 16 * RT * NC;
   __shared__ float red[R16_NW * E];
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, q = lane >> 4, p = lane & 15;
@@ -590,7 +601,10 @@ __global__ void __launch_bounds__(64 * R16_NW) lora_rows16_kernel(int M, int K, 
     for (int w = 0; w < R16_NW; w++) v += red[w * E + e];
     const int rr = e / NC, c = e % NC, r2 = m0 + rr;
     if (gridDim.y == 1) {
-      if (r2 < M && c < n) C[(long long)r2 * ldc + c] = alpha * v;
+      if (r2 < M && c < n) {
+        C[(long long)r2 * ldc + c] = alpha * v;
+        if (uo.p) put_u(uo, sg.r, r2, c, alpha * v, xh.rinv[r2]);
+      }
     } else {
       part[((long long)blockIdx.y * gridDim.x + blockIdx.x) * E + e] = v;
     }
@@ -729,11 +743,11 @@ void launch_rows_jobs(long long M, int NJ, int n, const RowsJobK& j0, const Rows
 }
 }  // namespace
 
-void launch_lora_rows(long long M, long long K, float alpha, const float* X, long long ldx, const float* Bt,
+bool launch_lora_rows(long long M, long long K, float alpha, const float* X, long long ldx, const float* Bt,
                       long long ldb, const RowsSeg& sg, float* C, long long ldc, float* ws, size_t ws_bytes,
-                      hipStream_t st, HIn xh, B16 b16) {
+                      hipStream_t st, HIn xh, B16 b16, UOut uo) {
   const int n = sg.nt * sg.r;
-  if (M <= 0 || n <= 0) return;
+  if (M <= 0 || n <= 0) return false;
   HOS_REQUIRE(n <= 96 && sg.nt >= 1 && sg.nt <= 4, HOS_E_INVALID, "lora_rows: n = nt·r must be <= 96");
   // fp16 path: 16-byte rows and segments on 8-element bounds (otherwise the f32 kernels, reading xh)
   bool f16 = xh.hi && xh.lo && b16.hi && b16.lo && b16.sc && K % 32 == 0 && ldx % 8 == 0 && ldb % 8 == 0 &&
@@ -752,7 +766,7 @@ void launch_lora_rows(long long M, long long K, float alpha, const float* X, lon
 #define ROWS16(NJV, RTV)                                                                                   \
   case NJV * 8 + RTV:                                                                                      \
     lora_rows16_kernel<NJV, RTV><<<grid, 64 * R16_NW, 0, st>>>((int)M, (int)K, kchunk, alpha, xh, ldx, b16, ldb, sg, \
-                                                               C, ldc, ws);                                \
+                                                               C, ldc, ws, uo);                            \
     break;
     switch (NJ * 8 + RT) {
       ROWS16(1, 1) ROWS16(2, 1) ROWS16(3, 1) ROWS16(4, 1) ROWS16(5, 1) ROWS16(6, 1)
@@ -766,10 +780,10 @@ void launch_lora_rows(long long M, long long K, float alpha, const float* X, lon
     if (S > 1) {
       const long long tot = (long long)gx * rb * NJ * 16;
       const RowsRed rd{ws, S, alpha, C, ldc};
-      lora_rows_reduce<<<ceil_div_i(tot, 256), 256, 0, st>>>(gx, rb, NJ * 16, (int)M, n, rd, rd);
+      lora_rows_reduce<<<ceil_div_i(tot, 256), 256, 0, st>>>(gx, rb, NJ * 16, (int)M, n, rd, rd, uo, sg.r, xh.rinv);
       HOS_HIP_CHECK(hipGetLastError());
     }
-    return;
+    return uo.p != nullptr;
   }
   HOS_REQUIRE(K % 4 == 0 && ldx % 4 == 0 && ldb % 4 == 0 && ((uintptr_t)Bt & 15) == 0 &&
                   (xh.hi ? (((uintptr_t)xh.hi & 7) == 0 && ((uintptr_t)xh.lo & 7) == 0 && xh.rinv)
@@ -784,7 +798,7 @@ void launch_lora_rows(long long M, long long K, float alpha, const float* X, lon
     const dim3 gw((unsigned)ceil_div_i(M, 16), (unsigned)((n + 15) / 16));
     lora_rows_wide_kernel<1><<<gw, 64 * ROWS_WIDE_NW, 0, st>>>((int)M, (int)K, alpha, X, ldx, Bt, ldb, sg, C, ldc, xh);
     HOS_HIP_CHECK(hipGetLastError());
-    return;
+    return false;
   }
   const int gx = ceil_div_i(M, 32);
   int S = 0, kchunk = 0;
@@ -793,6 +807,7 @@ void launch_lora_rows(long long M, long long K, float alpha, const float* X, lon
   HOS_REQUIRE(S == 1 || (size_t)S * gx * 32 * NJ * 16 * 4 <= ws_bytes, HOS_E_INVALID, "lora_rows: workspace too small");
   const RowsJobK jb{(int)K, kchunk, S, alpha, X, ldx, Bt, ldb, sg, C, ldc, ws};
   launch_rows_jobs(M, NJ, n, jb, jb, 1, xh, st);
+  return false;
 }
 
 // Two independent f32 rows products over the same rows (u = x·A and du = s·dy·Bᵀ of the LoRA branch op) in one

@@ -30,11 +30,19 @@ struct RowsSeg {
   int kbeg[4] = {0, 0, 0, 0}, kend[4] = {0, 0, 0, 0};
   long long boff[4] = {0, 0, 0, 0};
 };
+// The product also as the plane GEMM's rank factor (GemmEpi::Uf): bf16 hi at p, lo at p + lo, divided by the row's
+// rinv, column j of slot t at slot·t + j (row stride ld). p == nullptr: not wanted.
+struct UOut {
+  __bf16* p = nullptr;
+  long long ld = 0, lo = 0;
+  int slot = 0;
+};
 // C[m, j] = α·Σ_k X[m, k]·B(j, k) for m < M, j < nt·r. X rows 16-byte aligned, K % 4 == 0. xh.hi set: X is
 // that operand (row stride ldx, 8-byte aligned rows) and the f32 pointer is not read.
-void launch_lora_rows(long long M, long long K, float alpha, const float* X, long long ldx, const float* Bt,
+// Returns whether uo was written too (the fp16 path writes it).
+bool launch_lora_rows(long long M, long long K, float alpha, const float* X, long long ldx, const float* Bt,
                       long long ldb, const RowsSeg& sg, float* C, long long ldc, float* ws, size_t ws_bytes,
-                      hipStream_t st, HIn xh = HIn{}, B16 b16 = B16{});
+                      hipStream_t st, HIn xh = HIn{}, B16 b16 = B16{}, UOut uo = UOut{});
 // The arguments of one f32 launch_lora_rows product.
 struct RowsCall {
   long long K;

@@ -102,6 +102,7 @@ struct hos_peft {
   QWeight tok, out;
   bool out_set = false;
   float* out_norm = nullptr;
+  void* plane_arena = nullptr;  // fp16 planes of the frozen weights (QWeight::pl points into it)
   bool stacks_dirty = true;  // a projection or bias changed since the stacked copies were built
 
   // LoRA arena offsets (floats): per (layer, group) the stacked At and Bcat blocks; per (layer, target)
@@ -124,6 +125,15 @@ struct hos_peft {
   std::vector<int> scA, scB;
   SplitRow* split_tab = nullptr;
   int n_split = 0;
+  // The same factors as the plane GEMMs' rank terms read them (GemmEpi::Lf), per (layer, group) Bcat (forward) and At
+  // (dX), from the table rank_tab; and u / du as their other side (Uf), one buffer per group and direction, written by
+  // the rows products of a group and read by its GEMMs (uready: written for the layer in progress).
+  __bf16* rfrag = nullptr;
+  RankItem* rank_tab = nullptr;
+  int n_rank = 0;
+  std::vector<long long> offLf;  // [(layer·4 + group)·2 + dX]
+  __bf16* uplane[4][2] = {};
+  bool uready[4][2] = {};
   long long nfac = 0;
   uint64_t adam_t = 0;
 
@@ -324,11 +334,35 @@ struct hos_peft {
   // column of target t's output inside the buffer its group's projections write (fused q|k|v, gate|up)
   int ycol(int t) const { return t == TK ? qd : (t == TV ? qd + kvd : (t == TU ? F : 0)); }
 
-  void lora_rows(const char* cls, long long M, long long K, float alpha, const float* X, long long ldx,
+  bool lora_rows(const char* cls, long long M, long long K, float alpha, const float* X, long long ldx,
                  const float* Bt, long long ldb, const RowsSeg& sg, float* C, long long ldc, HIn xh = HIn{},
-                 B16 b16 = B16{}) {
+                 B16 b16 = B16{}, UOut uo = UOut{}) {
     Scope s(this, cls, 2.0 * M * K * sg.nt * sg.r, 4.0 * (M * K + (double)M * sg.nt * sg.r));
-    launch_lora_rows(M, K, alpha, X, ldx, Bt, ldb, sg, C, ldc, ws, ws_bytes, st, xh, b16);
+    return launch_lora_rows(M, K, alpha, X, ldx, Bt, ldb, sg, C, ldc, ws, ws_bytes, st, xh, b16, uo);
+  }
+  // Row width of a group's Uf planes: 32 columns per target forward (each target's own factor), the stacked rank dX.
+  int uwidth(int g, bool dxdir) const { return dxdir ? (gcount(g) * r + 31) / 32 * 32 : 32 * gcount(g); }
+  UOut uout(int g, bool dxdir) const {
+    UOut o;
+    o.p = uplane[g][dxdir];
+    o.ld = uwidth(g, dxdir);
+    o.lo = (long long)Mmax * o.ld;
+    o.slot = dxdir ? r : 32;
+    return o;
+  }
+  // Point a rank term at the planes of its group (the whole group, or the one target t of a forward launch).
+  void rank_planes(GemmEpi& e, int l, int g, bool dxdir, int t = -1) const {
+    if (!uready[g][dxdir]) return;
+    const int nrs = dxdir ? uwidth(g, true) / 32 : 1;
+    long long nb0 = 0;
+    if (t >= 0) {
+      if (dxdir ? gcount(g) != 1 : bcol(t) % 16 != 0) return;
+      if (!dxdir) nb0 = bcol(t) / 16;
+    }
+    e.Uf = uplane[g][dxdir] + (t >= 0 && !dxdir ? 32 * slot(t) : 0);
+    e.ldf = uwidth(g, dxdir);
+    e.ulo = (long long)Mmax * e.ldf;
+    e.Lf = rfrag + offLf[(l * 4 + g) * 2 + dxdir] + nb0 * nrs * 1024;
   }
   // The fp16 operand of the activation the current GEMM reads (when it carries the residual plane) and the
   // factor split of a group's At (a) or Bcat: the LoRA rows products then run on fp16 MFMA.
@@ -342,6 +376,7 @@ struct hos_peft {
     if (n_split == 0) return;
     Scope s(this, "convert", 0, 8.0 * nfac);
     launch_split_rows16(split_tab, n_split, P, P16h, P16l, psc, st);
+    launch_rank_frags(rank_tab, n_rank, P, rfrag, st);
   }
   void lora_cols(const char* cls, long long M, int ns, float alpha, const float* Sm, long long lds, const float* Gm,
                  long long ldg, const ColsSeg& sg, float* C, long long scj, long long scc) {
@@ -365,8 +400,8 @@ struct hos_peft {
       sg.kend[i] = in;
       sg.boff[i] = (long long)i * r * in;
     }
-    lora_rows("lora_down", M, in, 1.0f, x, ldx, P + offAg[l * 4 + g], in, sg, act[l].u + ucol(first), NT * r, xh,
-              xh.hi ? fac16(l, g, true) : B16{});
+    uready[g][0] = lora_rows("lora_down", M, in, 1.0f, x, ldx, P + offAg[l * 4 + g], in, sg, act[l].u + ucol(first),
+                             NT * r, xh, xh.hi ? fac16(l, g, true) : B16{}, uout(g, false));
   }
   // Epilogue term y += s·u_t·B_t of the base forward GEMM: L(j, n) = Bcat[j·bw + bcol(t) + n]
   GemmEpi up_epi(int l, int t) {
@@ -379,6 +414,7 @@ struct hos_peft {
     e.sln = 1;
     e.rank = r;
     e.scale = lscale;
+    rank_planes(e, l, group_of(t), false, t);
     return e;
   }
   // A group's projections as one stacked GEMM: possible when its targets are all adapted or none is (the
@@ -407,6 +443,7 @@ struct hos_peft {
     e.ustep = r;
     e.ub0 = out_dim(t0);
     e.ub1 = g == 0 ? out_dim(TQ) + out_dim(TK) : 1 << 30;
+    rank_planes(e, l, g, false);
     return e;
   }
   // dX epilogue of a stacked group: dx_in += [du_1 … du_G]·[A_1ᵀ; …; A_Gᵀ], one rank-G·r term (At block).
@@ -420,6 +457,7 @@ struct hos_peft {
     e.sln = 1;
     e.rank = gcount(g) * r;
     e.scale = 1.0f;
+    rank_planes(e, l, g, true);
     return e;
   }
   // (Re)build the stacked copies of every layer (host side, before a step; never inside a capture).
@@ -443,8 +481,80 @@ struct hos_peft {
         HOS_HIP_CHECK(hipMemcpyAsync(w.bias_qkv + qd + kvd, w.bias[2], (size_t)kvd * 4, hipMemcpyDeviceToDevice, st));
       }
     }
+    build_plane_arena();
     HOS_HIP_CHECK(hipStreamSynchronize(st));
     stacks_dirty = false;
+  }
+  // Which form of a group the step's GEMMs take (forward / dX): the stacked weight or each projection on its own.
+  bool qkv_stacked(const LayerW& w, bool dxdir) const {
+    return w.qkv.q && group_uniform(0) && (dxdir ? gcount(0) * r <= 128 : !c.attn_bias || w.bias_qkv);
+  }
+  bool gu_stacked(const LayerW& w, bool dxdir) const {
+    return w.gu.q && group_uniform(2) && (!dxdir || gcount(2) * r <= 32);
+  }
+  // The fp16 planes of every weight the step multiplies by (planes.hip), in one allocation; a weight whose planes no
+  // longer fit (planes_fit) keeps the dequantizing GEMM.
+  void build_plane_arena() {
+    struct Item {
+      QWeight* w;
+      bool dx;
+      int planes, groups;
+      size_t bytes;
+    };
+    std::vector<Item> items;
+    size_t total = 0;
+    auto add = [&](QWeight& w, bool dxdir, int np, int groups = 1) {
+      if (!w.q || !plane_gemm_wanted(w, dxdir, np, Mmax, groups)) return;
+      const int n = planes_for(np);
+      const size_t b = planes_bytes(w, dxdir, n, groups);
+      if (!planes_fit(total + b)) return;
+      total += b;
+      items.push_back(Item{&w, dxdir, n, groups, b});
+    };
+    auto clear = [](QWeight& w) {
+      for (WPlanes& p : w.pl) p = WPlanes{};
+    };
+    for (LayerW& w : lw) {
+      for (QWeight& q : w.w) clear(q);
+      for (QWeight* q : {&w.xg, &w.xu, &w.xd, &w.xgu, &w.qkv, &w.gu}) clear(*q);
+    }
+    clear(tok);
+    clear(out);
+    if (plane_arena) (void)hipFree(plane_arena);
+    plane_arena = nullptr;
+    for (LayerW& w : lw)
+      for (bool dxdir : {false, true}) {
+        auto np = [&](int t) { const int o = dxdir ? tpd[t] : tpf[t]; return o ? o : (dxdir ? pd : pf); };
+        auto each = [&](bool stacked, QWeight& st_w, int t0, int t1) {
+          if (stacked) add(st_w, dxdir, np(t0));
+          else
+            for (int t = t0; t <= t1; t++) add(w.w[t], dxdir, np(t));
+        };
+        each(qkv_stacked(w, dxdir), w.qkv, TQ, TV);
+        add(w.w[TO], dxdir, np(TO));
+        if (E) {
+          if (w.xgu.q) add(w.xgu, dxdir, np(TG), E);
+          else
+            for (QWeight* q : {&w.xg, &w.xu}) add(*q, dxdir, np(TG), E);
+          add(w.xd, dxdir, np(TD), E);
+        } else {
+          each(gu_stacked(w, dxdir), w.gu, TG, TU);
+          add(w.w[TD], dxdir, np(TD));
+        }
+      }
+    for (bool dxdir : {false, true}) add(out_set ? out : tok, dxdir, dxdir ? phd : phf);
+    if (total == 0) return;
+    if (hipMalloc(&plane_arena, total) != hipSuccess) {
+      (void)hipGetLastError();
+      plane_arena = nullptr;
+      return;
+    }
+    char* p = (char*)plane_arena;
+    for (const Item& it : items) {
+      build_planes(*it.w, it.dx, it.planes, it.groups, (half_t*)p, st);
+      it.w->pl[it.dx] = WPlanes{(half_t*)p, it.planes, false};
+      p += it.bytes;
+    }
   }
   // Per-expert row interleave of two expert stacks of one encoding and width ([E·F][d] each): expert e's rows of a,
   // then its rows of b (the q and s arrays are row-major, so each expert's block of rows is one contiguous run of
@@ -516,8 +626,9 @@ struct hos_peft {
       rs.boff[i] = bcol(t);
     }
     const int w = bw(g);
-    lora_rows("lora_du", M, kspan, lscale, dy, ldy, P + offBg[l * 4 + g], w, rs, du_of(l) + ucol(first_adapted(g)),
-              NT * r, dyh, dyh.hi ? fac16(l, g, false) : B16{});
+    uready[g][1] = lora_rows("lora_du", M, kspan, lscale, dy, ldy, P + offBg[l * 4 + g], w, rs,
+                             du_of(l) + ucol(first_adapted(g)), NT * r, dyh, dyh.hi ? fac16(l, g, false) : B16{},
+                             uout(g, true));
     pend_db = ColsJob{r, lscale, act[l].u, NT * r, dy, ldy, cs, G + offBg[l * 4 + g], w, 1, dy ? HIn{} : dyh};
     pend_group = g;
   }
@@ -532,6 +643,7 @@ struct hos_peft {
     e.sln = 1;
     e.rank = r;
     e.scale = 1.0f;
+    rank_planes(e, l, group_of(t), true, t);
     return e;
   }
   // [dA_1 … dA_G]ᵀ = ([du_1 … du_G])ᵀ·x, written straight into the stacked At layout, in one launch with the
@@ -706,7 +818,7 @@ struct hos_peft {
         xsrc = SplitSrc{};
       }
       lora_down(l, 0, a.xn1, d, M, hs_in());
-      if (w.qkv.q && group_uniform(0) && (!c.attn_bias || w.bias_qkv)) {
+      if (qkv_stacked(w, false)) {
         qfwd(w.qkv, hs, d, M, a.qkv, W3, c.attn_bias ? w.bias_qkv : nullptr, nullptr, 0, stacked_up_epi(l, 0),
              tpf[TQ]);
       } else {
@@ -740,7 +852,7 @@ struct hos_peft {
         continue;
       }
       lora_down(l, 2, a.xn2, d, M, hs_in());
-      if (w.gu.q && group_uniform(2)) {
+      if (gu_stacked(w, false)) {
         qfwd(w.gu, hs, d, M, a.gu, 2LL * F, nullptr, nullptr, 0, stacked_up_epi(l, 2), tpf[TG]);
       } else {
         qfwd(w.w[TG], hs, d, M, a.gu, 2LL * F, nullptr, nullptr, 0, up_epi(l, TG), tpf[TG]);
@@ -824,7 +936,7 @@ struct hos_peft {
         launch_swiglu_bwd(a.gu, dh, M, F, gu_f32 ? dgu : nullptr, hg, st);
       }
       if (gu_lora) lora_grad_b(l, 2, gu_f32 ? dgu : nullptr, 2LL * F, 2LL * F, M, HIn{hg.data, hg.lo, hg.rinv});
-      if (w.gu.q && group_uniform(2) && gcount(2) * r <= 32) {
+      if (gu_stacked(w, true)) {
         gsrc = deferred(true, w.gu, hg, 2LL * F, M, dxn, d, nullptr, stacked_down_epi(l, 2), tpd[TG]);
       } else {
         H16 hu = h16_offset(hg, F);
@@ -873,7 +985,7 @@ struct hos_peft {
       }
       if (c.qk_norm) to16(dq, W3, M, W3);
       lora_grad_b(l, 0, dq, W3, W3, M, hs_in());
-      if (w.qkv.q && group_uniform(0) && gcount(0) * r <= 128) {
+      if (qkv_stacked(w, true)) {
         // one dX GEMM over the stacked q|k|v contraction, the three LoRA terms as one rank-3r update
         qdx(w.qkv, hs, W3, M, dxn, d, 0, stacked_down_epi(l, 0), tpd[TQ]);
       } else {
@@ -1144,6 +1256,32 @@ struct hos_peft {
         P16h = alloc<_Float16>(nparams);
         P16l = alloc<_Float16>(nparams);
         psc = alloc<float>(tab.size());
+        std::vector<RankItem> items;
+        offLf.assign((size_t)L * 8, -1);
+        long long fo = 0;
+        for (int l = 0; l < L; l++)
+          for (int g = 0; g < 4; g++) {
+            if (offAg[l * 4 + g] < 0) continue;
+            for (int dxdir = 0; dxdir < 2; dxdir++) {
+              const int rank = dxdir ? gcount(g) * r : r, cols = dxdir ? in_dim(group_first(g)) : bw(g);
+              const int nrs = (rank + 31) / 32;
+              offLf[(l * 4 + g) * 2 + dxdir] = fo;
+              for (int nb = 0; nb < (cols + 15) / 16; nb++, fo += 1024LL * nrs)
+                items.push_back(RankItem{dxdir ? offAg[l * 4 + g] : offBg[l * 4 + g], fo, cols, rank, cols, nb,
+                                         dxdir ? 1.0f : lscale});
+            }
+          }
+        n_rank = (int)items.size();
+        rank_tab = alloc<RankItem>(items.size());
+        HOS_HIP_CHECK(hipMemcpy(rank_tab, items.data(), items.size() * sizeof(RankItem), hipMemcpyHostToDevice));
+        rfrag = alloc<__bf16>(fo);
+        for (int g = 0; g < 4; g++)
+          for (int dxdir = 0; dxdir < 2; dxdir++) {
+            if (gcount(g) == 0) continue;
+            const size_t n = 2 * (size_t)Mmax * uwidth(g, dxdir);
+            uplane[g][dxdir] = alloc<__bf16>(n);
+            launch_fill((float*)uplane[g][dxdir], (long long)(n / 2), 0.0f, st);  // the padding stays zero
+          }
       }
     }
     P = alloc<float>(nparams);
@@ -1319,6 +1457,8 @@ struct hos_peft {
     }
     free_qweight(tok);
     free_qweight(out);
+    if (plane_arena) (void)hipFree(plane_arena);
+    plane_arena = nullptr;
     for (void* p : allocs) (void)hipFree(p);
     allocs.clear();
   }

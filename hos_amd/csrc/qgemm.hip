@@ -106,6 +106,7 @@ void launch_any(bool dx, const QWeight& w, H16 a, long long lda, long long M, Ge
                 size_t ws_bytes, int passes, hipStream_t st) {
   if (M <= 0) return;
   HOS_REQUIRE(passes >= 1 && passes <= 5, HOS_E_INVALID, "qgemm: precision mode must be 1 to 5");
+  if (launch_plane_gemm(dx, w, a, lda, M, epi, ws, ws_bytes, passes, st)) return;
   switch (w.type) {
     case GGUF_Q8_0: qgemm_launch_q8(dx, passes, w, a, lda, M, epi, ws, ws_bytes, st); break;
     case GGUF_Q4_K: qgemm_launch_q4k(dx, passes, w, a, lda, M, epi, ws, ws_bytes, st); break;
@@ -132,6 +133,7 @@ void launch_qgemm_grouped(bool dx, const QWeight& w, GroupSched gs, H16 a, long 
                           hipStream_t st) {
   HOS_REQUIRE(passes >= 1 && passes <= 5, HOS_E_INVALID, "qgemm: precision mode must be 1 to 5");
   if (gs.max_tiles <= 0) return;
+  if (launch_plane_gemm_grouped(dx, w, gs, a, lda, epi, passes, st)) return;
   switch (w.type) {
     case GGUF_Q8_0: qgemm_grouped_q8(dx, passes, w, gs, a, lda, epi, st); break;
     case GGUF_Q4_K: qgemm_grouped_q4k(dx, passes, w, gs, a, lda, epi, st); break;
