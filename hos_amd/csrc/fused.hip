@@ -713,6 +713,125 @@ __global__ void __launch_bounds__(RB) ce_kernel(const float* __restrict__ logits
   if (threadIdx.x == 0) rinv[row] = ldexpf(1.0f, -e);
 }
 
+// The same with the plain f32 gradient (the op-level entry, the full finetune), for wide rows: HBM bound, so the logits
+// are read from it once. One workgroup of 16 waves per CU holds the row from the statistics to the gradient — 192 KB of
+// it in registers, 144 KB in LDS — and what is left of a wider row is read again last in, first out, out of the caches
+// (256 rows' remainders fit the last-level cache; 2048 rows at once, as in ce_kernel, do not). Gradient stores bypass the
+// caches. 2048 × 151936 on the MI355X: 818 -> 624 µs (2.49 GB; a copy of that size takes 508).
+constexpr int CEB = 1024;
+template <int W>
+struct alignas(4 * W) CeVec {
+  float v[W];
+};
+template <int W>
+__global__ void __launch_bounds__(CEB) ce_wide_kernel(const float* __restrict__ logits, int V,
+                                                      const int32_t* __restrict__ targets, float gscale,
+                                                      float* __restrict__ row_loss, float* __restrict__ dl32) {
+  using T = CeVec<W>;
+  constexpr int NR = (W == 4 ? 48 : 16) / W, NL = 36 / W;  // vectors per thread in registers, in LDS
+  __shared__ T keep[NL][CEB];
+  __shared__ float rm[CEB / 64], rs[CEB / 64];
+  const int row = blockIdx.x, tid = threadIdx.x, n = V / W;
+  const T* lr = reinterpret_cast<const T*>(logits + (long long)row * V);
+  T none;
+#pragma unroll
+  for (int e = 0; e < W; e++) none.v[e] = -INFINITY;
+  float m = -INFINITY, sum = 0.0f;
+  // (the max's own term is 1 without an exponential: +inf has one, too)
+  auto term = [&](float x) { return x == m ? 1.0f : expf(x - m); };
+  auto add = [&](const T& x) {
+    float mx = x.v[0];
+#pragma unroll
+    for (int e = 1; e < W; e++) mx = fmaxf(mx, x.v[e]);
+    if (mx > m) {
+      sum *= expf(m - mx);
+      m = mx;
+    }
+#pragma unroll
+    for (int e = 0; e < W; e++) sum += term(x.v[e]);
+  };
+  T x[NR];
+#pragma unroll
+  for (int j = 0; j < NR; j++) x[j] = tid + CEB * j < n ? lr[tid + CEB * j] : none;
+#pragma unroll
+  for (int j = 0; j < NR; j++)
+#pragma unroll
+    for (int e = 0; e < W; e++) m = fmaxf(m, x[j].v[e]);
+#pragma unroll
+  for (int j = 0; j < NR; j++) {
+    if (tid + CEB * j < n)
+#pragma unroll
+      for (int e = 0; e < W; e++) sum += term(x[j].v[e]);
+    __builtin_amdgcn_sched_barrier(0);  // no interleaving of the vectors: it costs more registers than there are
+  }
+#pragma unroll 1
+  for (int k = 0; k < NL; k += 3) {
+    T y[3];
+#pragma unroll
+    for (int u = 0; u < 3; u++) {
+      const int c = tid + CEB * (NR + k + u);
+      y[u] = c < n ? lr[c] : none;
+    }
+#pragma unroll
+    for (int u = 0; u < 3; u++)
+      if (tid + CEB * (NR + k + u) < n) {
+        keep[k + u][tid] = y[u];
+        add(y[u]);
+      }
+  }
+  const int c0 = tid + CEB * (NR + NL);
+  for (int c = c0; c < n; c += 4 * CEB) {
+    T y[4];
+#pragma unroll
+    for (int u = 0; u < 4; u++) y[u] = c + CEB * u < n ? lr[c + CEB * u] : none;
+#pragma unroll
+    for (int u = 0; u < 4; u++)
+      if (c + CEB * u < n) add(y[u]);
+  }
+  for (int o = 32; o > 0; o >>= 1) sm_merge(m, sum, __shfl_xor(m, o), __shfl_xor(sum, o));
+  if ((tid & 63) == 0) {
+    rm[tid >> 6] = m;
+    rs[tid >> 6] = sum;
+  }
+  __syncthreads();
+  m = rm[0];
+  sum = rs[0];
+#pragma unroll
+  for (int w = 1; w < CEB / 64; w++) sm_merge(m, sum, rm[w], rs[w]);
+  const int t = targets[row];
+  if (tid == 0) row_loss[row] = -logf(fmaxf(expf(logits[(long long)row * V + t] - m) / sum, 1e-12f));
+  const float inv = 1.0f / sum;
+  T* out = reinterpret_cast<T*>(dl32 + (long long)row * V);
+  auto grad = [&](const T& z, int c) {
+#pragma unroll
+    for (int e = 0; e < W; e++) {
+      float p = expf(z.v[e] - m) * inv;
+      if (W * c + e == t) p -= 1.0f;
+      __builtin_nontemporal_store(p * gscale, &out[c].v[e]);
+    }
+  };
+  if (c0 < n) {
+    for (int c = c0 + (n - 1 - c0) / (4 * CEB) * (4 * CEB); c >= c0; c -= 4 * CEB) {
+      T y[4];
+#pragma unroll
+      for (int u = 0; u < 4; u++) y[u] = c + CEB * u < n ? lr[c + CEB * u] : none;
+#pragma unroll
+      for (int u = 0; u < 4; u++)
+        if (c + CEB * u < n) grad(y[u], c + CEB * u);
+    }
+  }
+#pragma unroll 1
+  for (int k = 0; k < NL; k++) {
+    if (tid + CEB * (NR + k) < n) grad(keep[k][tid], tid + CEB * (NR + k));
+    __builtin_amdgcn_sched_barrier(0);
+  }
+#pragma unroll
+  for (int j = 0; j < NR; j++) {
+    if (tid + CEB * j < n) grad(x[j], tid + CEB * j);
+    __builtin_amdgcn_sched_barrier(0);
+  }
+}
+
 // loss = Σ_b (Σ_t term[b,t] / T) · (1/B), in sequence order (src/main.rs:2588-2596). Each sequence is
 // staged in LDS by the whole workgroup and summed in order by one thread.
 __global__ void __launch_bounds__(256) loss_reduce_kernel(const float* __restrict__ row_loss, int B, int T,
@@ -934,8 +1053,20 @@ void launch_swiglu_bwd(const float* gu, const float* dh, int M, int F, float* dg
     swiglu_bwd_kernel<<<M, RB, 0, st>>>(gu, dh, F, dgu, out.data, out.lo, out.rinv);
   HOS_HIP_CHECK(hipGetLastError());
 }
+// Rows from which ce_wide_kernel is the faster one: a row a CU pays from 24k columns on; below, only while the rows are
+// few (2048 rows: 32000 columns 188 -> 155 µs, 16384 69 against 104; 300 rows: 16384 34 -> 27, 151936 321 -> 142).
+static bool ce_wide(int M, int V) { return V >= 24576 || (V >= 16384 && M <= 512); }
+
 void launch_ce(const float* logits, int M, int V, const int32_t* targets, float gscale, float* row_loss, H16 dl,
                hipStream_t st, float* dl32, const float2* rstat) {
+  if (dl32 && !rstat && ce_wide(M, V)) {
+    if (V % 4 == 0 && ((uintptr_t)logits & 15) == 0 && ((uintptr_t)dl32 & 15) == 0)
+      ce_wide_kernel<4><<<M, CEB, 0, st>>>(logits, V, targets, gscale, row_loss, dl32);
+    else
+      ce_wide_kernel<1><<<M, CEB, 0, st>>>(logits, V, targets, gscale, row_loss, dl32);
+    HOS_HIP_CHECK(hipGetLastError());
+    return;
+  }
   ce_kernel<<<M, RB, 0, st>>>(logits, V, targets, gscale, row_loss, dl.data, dl.lo, dl.rinv, dl32, rstat,
                               (V + 63) / 64);
   HOS_HIP_CHECK(hipGetLastError());

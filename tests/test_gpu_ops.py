@@ -152,6 +152,33 @@ def test_cross_entropy(gpu, rows, V):
         a.free()
 
 
+# Rows wide enough for the one-workgroup-per-row kernel: whole and ragged vectors, the last column of what it holds in
+# registers (49152) and in LDS (86016; 53248 for widths that are no multiple of 4), and one past them. Against float64:
+# p is one expf and two products of the f32 logits off (~2e-7), the row's sum of up to 1e5 terms ~1e-7.
+@pytest.mark.parametrize("rows,V", [(5, 24576), (3, 24577), (2, 49156), (2, 53249), (2, 86016), (3, 86020), (2, 102401)])
+def test_cross_entropy_wide_rows(gpu, rows, V):
+    print(f"cross_entropy wide {rows} x {V}", flush=True)
+    rng = np.random.default_rng(V)
+    lg = (rng.standard_normal((rows, V)) * 2).astype(np.float32)
+    tg = rng.integers(0, V, rows).astype(np.int32)
+    tg[-1] = V - 1
+    lg[0, 0], lg[1, V - 1] = 30.0, -np.inf  # a row that one column takes, a masked column
+    gs = 1.0 / rows
+    ld, td, rl, dl = gpu.to_dev(lg), gpu.to_dev(tg), gpu.empty_dev((rows,)), gpu.empty_dev((rows, V))
+    gpu.op("cross_entropy", ld, rows, V, td, gs, rl, dl)
+    x = lg.astype(np.float64)
+    p = np.exp(x - x.max(1, keepdims=True))
+    p /= p.sum(1, keepdims=True)
+    loss = -np.log(np.maximum(p[np.arange(rows), tg], 1e-12))
+    p[np.arange(rows), tg] -= 1
+    got_l, got = rl.get(), dl.get()
+    for a in (ld, td, rl, dl):
+        a.free()
+    assert np.abs(got_l - loss).max() <= 2e-6 * np.abs(loss).max()
+    assert np.linalg.norm(got - p * gs) <= 1e-6 * np.linalg.norm(p * gs)
+    assert np.abs(got - p * gs).max() <= 2e-6 * gs
+
+
 def test_adamw_bit_exact(gpu):
     n = 10007
     print("adamw", flush=True)
