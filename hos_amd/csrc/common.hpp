@@ -76,6 +76,9 @@ struct WPlanes {
   half_t* p = nullptr;
   int planes = 0;  // 1: hi only, 2: hi and lo
   bool owned = false;
+  // Set: p holds the exact integer codes of a Q8_0-layout weight (one plane, forward) and this their block scales,
+  // 16 columns of one 32-deep step together: (nb, ks, column).
+  const float* scale = nullptr;
 };
 
 struct QWeight {

@@ -184,11 +184,22 @@ void launch_qgemm_fwd(const QWeight& w, H16 a, long long lda, long long M, GemmE
 void launch_qgemm_dx(const QWeight& w, H16 a, long long lda, long long M, GemmEpi epi, float* ws, size_t ws_bytes,
                      int passes, hipStream_t st);
 // ---- planes.hip / plane_gemm.hip ----
-// Planes a launch in this precision mode reads (hi, or hi and lo).
-inline int planes_for(int passes) { return passes >= 3 ? 2 : 1; }
-size_t planes_bytes(const QWeight& w, bool dx, int planes, int groups);
+// What a launch in this precision mode reads: 1 the hi plane, 2 hi and lo, kPlaneCodes the integer codes and scales.
+constexpr int kPlaneCodes = 5;
+inline int plane_kind(const QWeight& w, bool dx, int passes) {
+  if (passes == 5 && !dx && w.type == GGUF_Q8_0) return kPlaneCodes;
+  return passes >= 3 ? 2 : 1;
+}
+// Whether planes serve a launch: mode 5 runs on the codes or, as its three-product form, on hi and lo.
+inline bool has_planes(const WPlanes& p, bool dx, int passes) {
+  return p.scale ? passes == 5 && !dx : p.planes >= (passes >= 3 ? 2 : 1);
+}
+// Whether a three-product launch of M rows takes plane_chain_kernel (a model of that many rows at most then keeps hi
+// and lo planes instead of codes).
+bool plane_chain(long long M, long long N, long long C);
+size_t planes_bytes(const QWeight& w, bool dx, int kind, int groups);
 // Dequantize w into planes at dst (groups: experts stacked in w, each laid out on its own).
-void build_planes(const QWeight& w, bool dx, int planes, int groups, half_t* dst, hipStream_t st);
+WPlanes build_planes(const QWeight& w, bool dx, int kind, int groups, half_t* dst, hipStream_t st);
 // Whether a launch of M rows on this weight takes the plane GEMM once the planes are there (groups > 1: grouped).
 bool plane_gemm_wanted(const QWeight& w, bool dx, int passes, long long M, int groups = 1);
 // Whether planes of this size may be allocated: they never take the card's free memory below half of its total, so

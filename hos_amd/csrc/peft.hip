@@ -498,14 +498,15 @@ struct hos_peft {
     struct Item {
       QWeight* w;
       bool dx;
-      int planes, groups;
+      int kind, groups;
       size_t bytes;
     };
     std::vector<Item> items;
     size_t total = 0;
     auto add = [&](QWeight& w, bool dxdir, int np, int groups = 1) {
       if (!w.q || !plane_gemm_wanted(w, dxdir, np, Mmax, groups)) return;
-      const int n = planes_for(np);
+      int n = plane_kind(w, dxdir, np);
+      if (n == kPlaneCodes && groups == 1 && plane_chain(Mmax, w.rows, w.cols)) n = 2;
       const size_t b = planes_bytes(w, dxdir, n, groups);
       if (!planes_fit(total + b)) return;
       total += b;
@@ -551,8 +552,7 @@ struct hos_peft {
     }
     char* p = (char*)plane_arena;
     for (const Item& it : items) {
-      build_planes(*it.w, it.dx, it.planes, it.groups, (half_t*)p, st);
-      it.w->pl[it.dx] = WPlanes{(half_t*)p, it.planes, false};
+      it.w->pl[it.dx] = build_planes(*it.w, it.dx, it.kind, it.groups, (half_t*)p, st);
       p += it.bytes;
     }
   }

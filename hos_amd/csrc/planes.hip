@@ -40,6 +40,31 @@ __global__ void __launch_bounds__(256) build_fwd_kernel(QWeightView w, int plane
   }
 }
 
+// Mode 5's codes, laid out as the forward planes (one plane), and their scales.
+__global__ void __launch_bounds__(256) build_codes_kernel(QWeightView w, long long er, long long Np, int KT, long long groups,
+                                                          _Float16* __restrict__ dst, float* __restrict__ scale) {
+  const long long i = (long long)blockIdx.x * 256 + threadIdx.x;
+  const long long n = i % Np, u = i / Np, ks = u % KT, g = u / KT;
+  if (g >= groups) return;
+  __attribute__((aligned(16))) _Float16 v[32];
+  float sc = 0.0f;
+  if (n < er) {
+    const long long e = (g * er + n) * w.cols + 32 * ks;
+    Run<GGUF_Q8_0, 32> r;
+    run_load<GGUF_Q8_0, 32>((const uint8_t*)w.q + e, w.s + (e >> 5), r);
+    sc = r.s[0].x;
+    run_store<GGUF_Q8_0, 32, false, true>(r, v, 0);
+  } else {
+#pragma unroll
+    for (int q = 0; q < 32; q++) v[q] = (_Float16)0.0f;
+  }
+  const long long f = (g * (Np >> 4) + (n >> 4)) * KT + ks;
+  _Float16* d = dst + f * 512 + (n & 15) * 8;
+#pragma unroll
+  for (int q = 0; q < 4; q++) *(h8*)(d + q * 128) = *(const h8*)(v + 8 * q);
+  scale[f * 16 + (n & 15)] = sc;
+}
+
 // dX: the contraction runs down the rows, so a workgroup turns 32 rows × 256 columns round in LDS: a thread per run in,
 // then fragment pieces (8 rows of a column) out.
 template <uint32_t QT>
@@ -176,27 +201,41 @@ static void plane_dims(const QWeight& w, bool dx, int groups, long long* er, lon
   *C = dx ? *er : w.cols;
 }
 
-size_t planes_bytes(const QWeight& w, bool dx, int planes, int groups) {
+// 1 KB fragments of one plane.
+static size_t plane_frags(const QWeight& w, bool dx, int groups) {
   long long er, N, C;
   plane_dims(w, dx, groups, &er, &N, &C);
-  return (size_t)groups * ((N + 15) / 16) * (C / 32) * 1024 * planes;
+  return (size_t)groups * ((N + 15) / 16) * (C / 32);
 }
 
-void build_planes(const QWeight& w, bool dx, int planes, int groups, half_t* dst, hipStream_t st) {
+size_t planes_bytes(const QWeight& w, bool dx, int kind, int groups) {
+  return plane_frags(w, dx, groups) * (kind == kPlaneCodes ? 1024 + 64 : 1024 * kind);
+}
+
+WPlanes build_planes(const QWeight& w, bool dx, int kind, int groups, half_t* dst, hipStream_t st) {
   long long er, N, C;
   plane_dims(w, dx, groups, &er, &N, &C);
-  HOS_REQUIRE(w.rows % groups == 0 && C % 32 == 0 && w.cols % 32 == 0 && (long long)groups * (er / 32) < 65536 * (dx ? 1LL : 1LL << 32),
-              HOS_E_INVALID, "planes: contraction must be a multiple of 32");
+  HOS_REQUIRE(w.rows % groups == 0 && C % 32 == 0 && w.cols % 32 == 0 && (!dx || groups * (er / 32) < 65536), HOS_E_INVALID,
+              "planes: contraction must be a multiple of 32");
+  if (kind == kPlaneCodes) {
+    HOS_REQUIRE(!dx && w.type == GGUF_Q8_0, HOS_E_INVALID, "planes: integer codes are for forward Q8_0 weights");
+    float* scale = (float*)(dst + plane_frags(w, dx, groups) * 512);
+    const long long Np = (er + 15) / 16 * 16, KT = w.cols / 32;
+    build_codes_kernel<<<ceil_div(Np * KT * groups, 256), 256, 0, st>>>(view(w), er, Np, (int)KT, groups, dst, scale);
+    HOS_HIP_CHECK(hipGetLastError());
+    return WPlanes{dst, 1, false, scale};
+  }
   switch (w.type) {
-    case GGUF_Q8_0: build_typed<GGUF_Q8_0>(w, dx, planes, groups, dst, st); break;
-    case GGUF_Q4_K: build_typed<GGUF_Q4_K>(w, dx, planes, groups, dst, st); break;
-    case GGUF_Q6_K: build_typed<GGUF_Q6_K>(w, dx, planes, groups, dst, st); break;
-    case GGUF_Q5_K: build_typed<GGUF_Q5_K>(w, dx, planes, groups, dst, st); break;
-    case GGUF_F16: build_typed<GGUF_F16>(w, dx, planes, groups, dst, st); break;
-    case GGUF_BF16: build_typed<GGUF_BF16>(w, dx, planes, groups, dst, st); break;
-    case GGUF_F32: build_typed<GGUF_F32>(w, dx, planes, groups, dst, st); break;
+    case GGUF_Q8_0: build_typed<GGUF_Q8_0>(w, dx, kind, groups, dst, st); break;
+    case GGUF_Q4_K: build_typed<GGUF_Q4_K>(w, dx, kind, groups, dst, st); break;
+    case GGUF_Q6_K: build_typed<GGUF_Q6_K>(w, dx, kind, groups, dst, st); break;
+    case GGUF_Q5_K: build_typed<GGUF_Q5_K>(w, dx, kind, groups, dst, st); break;
+    case GGUF_F16: build_typed<GGUF_F16>(w, dx, kind, groups, dst, st); break;
+    case GGUF_BF16: build_typed<GGUF_BF16>(w, dx, kind, groups, dst, st); break;
+    case GGUF_F32: build_typed<GGUF_F32>(w, dx, kind, groups, dst, st); break;
     default: throw Error(HOS_E_UNSUPPORTED_QUANT, "planes: unsupported quant type");
   }
+  return WPlanes{dst, kind, false, nullptr};
 }
 
 // Planes a context may allocate between two looks at the free memory (a look costs as much as building small planes).
@@ -210,8 +249,8 @@ bool planes_fit(size_t bytes) {
 
 void ensure_planes(QWeight& w, bool dx, int passes, long long M, size_t* credit, hipStream_t st) {
   WPlanes& p = w.pl[dx];
-  const int want = planes_for(passes);
-  if (p.planes >= want || !plane_gemm_wanted(w, dx, passes, M)) return;
+  const int want = plane_kind(w, dx, passes);
+  if (has_planes(p, dx, passes) || !plane_gemm_wanted(w, dx, passes, M)) return;
   // A capture records the build without running it: later eager launches would read planes that are not there yet.
   hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
   HOS_HIP_CHECK(hipStreamIsCapturing(st, &cs));
@@ -227,13 +266,21 @@ void ensure_planes(QWeight& w, bool dx, int passes, long long M, size_t* credit,
     (void)hipGetLastError();  // no planes then: the launch runs on the quantized weight
     return;
   }
-  if (p.owned) {  // hi only so far, and launches on the stream may still read it
+  if (p.owned) {  // another kind so far, and launches on the stream may still read it
     HOS_HIP_CHECK(hipStreamSynchronize(st));
     (void)hipFree(p.p);
   }
   *credit -= bytes;
-  p = WPlanes{(half_t*)d, want, true};
-  build_planes(w, dx, want, 1, p.p, st);
+  p = WPlanes{};
+  WPlanes q{(half_t*)d, 0, true, nullptr};
+  try {
+    q = build_planes(w, dx, want, 1, (half_t*)d, st);
+  } catch (...) {
+    (void)hipFree(d);
+    throw;
+  }
+  q.owned = true;
+  p = q;
 }
 
 }  // namespace hos

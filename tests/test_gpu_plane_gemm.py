@@ -1,4 +1,4 @@
-"""The plane GEMM (launches of 64 rows and more on a frozen weight) at the edges of its tiles: row counts around 16-row
+"""The plane GEMM (launches of 8 rows and more on a frozen weight) at the edges of its tiles: row counts around 16-row
 fragments and 32/64/128-row tiles, output widths around the 16-column fragments and the 128/256-column tiles,
 contractions of one slab, an odd number of slabs and long enough to be split, and rank-r terms of one, two and three
 32-rank steps, against the same product in float64.
@@ -29,6 +29,8 @@ def gpu():
 # (dx, type, rows, cols, t): forward output width rows over a contraction of cols, dX the other way round
 SHAPES = [
     (False, Q8_0, 16, 32, 64),       # one fragment, one slab
+    (False, Q8_0, 48, 288, 8),       # fewer rows than a fragment has, more steps than the small kernel has waves
+    (True, Q4_K, 1152, 256, 33),     # the longest contraction of the small kernel
     (False, Q8_0, 40, 96, 65),       # a ragged 16-column block, three slabs
     (False, Q4_K, 129, 256, 127),
     (False, Q6_K, 257, 512, 129),    # one column past a 256-column tile
@@ -86,3 +88,37 @@ def test_plane_gemm_rank_term(gpu, which, rank, ldu):
     gpu.set_gemm_passes(1)
     err = np.linalg.norm(y - (base + term))
     assert err <= 2e-6 * np.linalg.norm(base) + 2e-5 * np.linalg.norm(term)
+
+
+# contractions of one, nine and fifteen slabs, of two splits, of four with a short last one, and outputs past 512
+# workgroups of 16 rows
+@pytest.mark.parametrize("n,c", [(32, 64), (576, 576), (96, 960), (576, 1536), (64, 2240), (1536, 576)])
+@pytest.mark.parametrize("which,rank", [(0, 0), (1, 0), (0, 16), (1, 33)])
+def test_chain_sums_are_the_dequantizing_kernels(gpu, which, rank, n, c):
+    """Under 8 rows the dequantizing kernel runs; 64 rows have its tiles and splits: equal bit for bit."""
+    print(f"chain {n} x {c} which {which} rank {rank}", flush=True)
+    t = 64
+    rng = np.random.default_rng(n + c + rank)
+    rows, cols = (n, c) if which == 0 else (c, n)
+    raw = o.quantize(rng.standard_normal((rows, cols)).astype(np.float32) * np.float32(0.05), Q8_0)
+    x = rng.standard_normal((t, c)).astype(np.float32)
+    u = rng.standard_normal((t, max(rank, 1))).astype(np.float32)
+    lf = rng.standard_normal((max(rank, 1), n)).astype(np.float32)
+    gpu.set_gemm_passes(3)
+    gpu.upload_quant(0x79, raw, Q8_0, rows, cols)
+
+    def product(i, j):
+        if rank == 0:
+            return gpu.qgemm_dx(0x79, x[i:j], cols) if which else gpu.qgemm_fwd(0x79, x[i:j], rows)
+        xd, ud, ld, out = gpu.to_dev(x[i:j].copy()), gpu.to_dev(u[i:j].copy()), gpu.to_dev(lf), gpu.empty_dev((j - i, n))
+        gpu.op("qgemm_lora_dev", which, 0x79, xd, j - i, ud, rank, ld, n, 1, rank, 1.5, out)
+        y = out.get()
+        for a in (xd, ud, ld, out):
+            a.free()
+        return y
+
+    y = product(0, t)
+    parts = np.concatenate([product(i, min(i + 7, t)) for i in range(0, t, 7)])
+    gpu.evict(0x79)
+    gpu.set_gemm_passes(1)
+    np.testing.assert_array_equal(y, parts)
