@@ -35,9 +35,16 @@ namespace {
 constexpr int TB = 32;        // rows of one MFMA tile
 constexpr int NW = 4;         // waves per workgroup
 constexpr int BR = TB * NW;   // rows a workgroup owns
-// Wave groups splitting the streamed axis of a workgroup. Forward: three at head dim 64 (a third of the key range
-// each, 110 KB of LDS; measured 3-6% faster than two), two at 128 (three would need 204 KB). Backward: two, except
-// for head dim 128, whose accumulators need more than the 256 registers two waves per SIMD leave (they spill).
+// Wave groups splitting the streamed axis of a workgroup, for launches that would leave compute units idle. Forward:
+// three at head dim 64 (a third of the key range each, 110 KB of LDS; measured 3-6% faster than two), two at 128 (three
+// would need 204 KB). Backward: two, except for head dim 128, whose accumulators need more than the 256 registers two
+// waves per SIMD leave (they spill). The groups of a workgroup meet at one barrier a tile and so do the same thing at the same
+// time (the matrix unit 26-29% busy); where there are workgroups enough, one group each and two or three workgroups to a
+// compute unit (168 and 256 registers: four and three a SIMD spill, 125 -> 151 µs and 182 -> 236) overlap one's products with
+// another's softmax, and one's start and end with another's loop. Forward + dQ + dK/dV in µs, groups against none, head dim 64:
+// 8 × 1024 × 32 heads (2048 workgroups) 709 -> 544, 4 × 1024 × 32 366 -> 286, 6 × 512 × 32 (768) 192 -> 144; 448: 8 × 512 × 14
+// 124 -> 103, but 4 × 1024 × 14 175 -> 174 and 1 × 4096 × 14 631 -> 710; 224: 80 -> 83. Head dim 128 (forward only): 1024 workgroups
+// 145 -> 126, 512 74 -> 82. So from 768 workgroups on, and at head dim 64 from 384 where sequences are short (whole_axis).
 #ifndef HOS_ATT_LPT
 #define HOS_ATT_LPT 1
 #endif
@@ -296,7 +303,7 @@ struct TileLoaderQD {
 // streams its range through its own double-buffered LDS stages, and the groups' (m, l, O) merge in group order
 // through LDS at the end.
 template <int HD, int NG>
-__global__ void __launch_bounds__(256 * NG) attn_fwd_kernel(const __bf16* __restrict__ qh, const __bf16* __restrict__ ql,
+__global__ void __launch_bounds__(256 * NG, HD == 64 && NG == 1 ? 3 : 1) attn_fwd_kernel(const __bf16* __restrict__ qh, const __bf16* __restrict__ ql,
                                                             const __bf16* __restrict__ kh, const __bf16* __restrict__ kl,
                                                             const __bf16* __restrict__ vh, const __bf16* __restrict__ vl,
                                                             int T, int nh, int group, float* __restrict__ o,
@@ -432,7 +439,7 @@ __global__ void __launch_bounds__(256 * NG) attn_fwd_kernel(const __bf16* __rest
 // ---- dQ: a wave owns 32 queries; K and V tiles stream through LDS ----
 // NG wave groups split the key tiles as in the forward; their partial dQ sums add in group order at the end.
 template <int HD, int NG>
-__global__ void __launch_bounds__(256 * NG) attn_dq_kernel(const __bf16* __restrict__ qh, const __bf16* __restrict__ ql,
+__global__ void __launch_bounds__(256 * NG, HD == 64 ? 2 : 1) attn_dq_kernel(const __bf16* __restrict__ qh, const __bf16* __restrict__ ql,
                                                       const __bf16* __restrict__ kh, const __bf16* __restrict__ kl,
                                                       const __bf16* __restrict__ vh, const __bf16* __restrict__ vl,
                                                       const float* __restrict__ o, const float* __restrict__ dout,
@@ -503,10 +510,17 @@ __global__ void __launch_bounds__(256 * NG) attn_dq_kernel(const __bf16* __restr
       float ds[16];
 #pragma unroll
       for (int r = 0; r < 16; r++) {
-        const int key = k0 + kap(r, hl);
-        const float pv = (key > myq || key >= T || myq >= T) ? 0.0f : exp_shift(S[r], Lq2);
-        ds[r] = pv * (dP[r] - Dq);
+        S[r] = exp_shift(S[r], Lq2);
       }
+      if (kb == my_last) {  // the tile of the diagonal and the sequence's end
+#pragma unroll
+        for (int r = 0; r < 16; r++) {
+          const int key = k0 + kap(r, hl);
+          if (key > myq || key >= T || myq >= T) S[r] = 0.0f;
+        }
+      }
+#pragma unroll
+      for (int r = 0; r < 16; r++) ds[r] = S[r] * (dP[r] - Dq);
       // dQᵀ += Kᵀ·dSᵀ
 #pragma unroll
       for (int t = 0; t < 2; t++) {
@@ -560,7 +574,7 @@ __global__ void __launch_bounds__(256 * NG) attn_dq_kernel(const __bf16* __restr
 // order; with group == 1 it is written in place. NG wave groups split the query tiles into consecutive ranges;
 // their partial dK / dV sums add in group order at the end.
 template <int HD, int NG>
-__global__ void __launch_bounds__(256 * NG) attn_dkdv_kernel(const __bf16* __restrict__ qh, const __bf16* __restrict__ ql,
+__global__ void __launch_bounds__(256 * NG, HD == 64 ? 2 : 1) attn_dkdv_kernel(const __bf16* __restrict__ qh, const __bf16* __restrict__ ql,
                                                         const __bf16* __restrict__ kh, const __bf16* __restrict__ kl,
                                                         const __bf16* __restrict__ vh, const __bf16* __restrict__ vl,
                                                         const float* __restrict__ dout, long long ldo,
@@ -634,12 +648,16 @@ __global__ void __launch_bounds__(256 * NG) attn_dkdv_kernel(const __bf16* __res
       }
       float p[16], ds[16];
 #pragma unroll
-      for (int r = 0; r < 16; r++) {
-        const int q = q0 + kap(r, hl);
-        const float pv = (mykey > q || q >= T || mykey >= T) ? 0.0f : exp_shift(S[r], Lr[r]);
-        p[r] = pv;
-        ds[r] = pv * (dP[r] - Dr[r]);
+      for (int r = 0; r < 16; r++) p[r] = exp_shift(S[r], Lr[r]);
+      if (qt == my_first || qt == nqt - 1) {  // the tiles of the diagonal and the sequence's end
+#pragma unroll
+        for (int r = 0; r < 16; r++) {
+          const int q = q0 + kap(r, hl);
+          if (mykey > q || q >= T || mykey >= T) p[r] = 0.0f;
+        }
       }
+#pragma unroll
+      for (int r = 0; r < 16; r++) ds[r] = p[r] * (dP[r] - Dr[r]);
       // dVᵀ += dOᵀ·P, dKᵀ += Qᵀ·dS (Q carries the scale, so this is already dK)
 #pragma unroll
       for (int t = 0; t < 2; t++) {
@@ -700,18 +718,22 @@ __global__ void __launch_bounds__(256 * NG) attn_dkdv_kernel(const __bf16* __res
 
 // dK/dV of kv head g = Σ over its group's heads, in head order (deterministic).
 template <int HD>
-__global__ void attn_group_sum(const float* __restrict__ part, int M, int nh, int nkv, int group,
+__global__ void attn_group_sum(const float4* __restrict__ part, int M, int nh, int nkv, int group,
                                float* __restrict__ dkv, long long ldk, int kcol, int vcol) {
+  constexpr int V = 2 * HD / 4;  // one thread per 4 columns
   long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= (long long)M * nkv * 2 * HD) return;
-  int c = (int)(i % (2 * HD));
-  long long t = i / (2 * HD);
+  if (i >= (long long)M * nkv * V) return;
+  const int c = (int)(i % V);
+  long long t = i / V;
   int g = (int)(t % nkv);
   long long m = t / nkv;
-  float s = 0.0f;
-  for (int hh = 0; hh < group; hh++) s += part[(m * nh + g * group + hh) * 2 * HD + c];
-  int col = (c < HD ? kcol : vcol) + g * HD + (c % HD);
-  dkv[m * ldk + col] = s;
+  float4 s = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+  for (int hh = 0; hh < group; hh++) {
+    const float4 x = part[(m * nh + g * group + hh) * V + c];
+    s = make_float4(s.x + x.x, s.y + x.y, s.z + x.z, s.w + x.w);
+  }
+  const int col = (4 * c < HD ? kcol : vcol) + g * HD + (4 * c) % HD;
+  *reinterpret_cast<float4*>(dkv + m * ldk + col) = s;
 }
 
 // Plane pointers inside the caller's scratch: q, k, v, each hi then lo.
@@ -746,15 +768,27 @@ void split_qkv(const float* qkv, long long ld, int kcol, int vcol, int B, int T,
   HOS_HIP_CHECK(hipGetLastError());
 }
 
+// Whether a launch has workgroups enough to leave the streamed axis whole (NG = 1).
+template <int HD>
+bool whole_axis(int B, int T, int nh) {
+  const long long wgs = (long long)ceil_div(T, BR) * nh * B;
+  return wgs >= 768 || (HD == 64 && wgs >= 384 && T <= 512);
+}
+
 template <int HD>
 void attn_fwd_hd(const float* qkv, long long ld, int kcol, int vcol, int B, int T, int nh, int nkv, float* o,
                  long long ldo, float* lse, void* scratch, hipStream_t st, const float2* rope_tab, bool rope_neox) {
   const Planes P = planes_of(scratch, B, T, nh, nkv, HD);
   split_qkv<HD>(qkv, ld, kcol, vcol, B, T, nh, nkv, P, st, rope_tab, rope_neox);
   dim3 grid(ceil_div(T, BR), nh, B);
-  constexpr int NGF = fwd_groups<HD>();
-  attn_fwd_kernel<HD, NGF><<<grid, 256 * NGF, 0, st>>>(P.qh, P.ql, P.kh, P.kl, P.vh, P.vl, T, nh, nh / nkv, o,
-                                                             ldo, lse);
+  const auto run = [&](auto ng) {
+    constexpr int NG = decltype(ng)::value;
+    attn_fwd_kernel<HD, NG><<<grid, 256 * NG, 0, st>>>(P.qh, P.ql, P.kh, P.kl, P.vh, P.vl, T, nh, nh / nkv, o, ldo, lse);
+  };
+  if (whole_axis<HD>(B, T, nh))
+    run(std::integral_constant<int, 1>{});
+  else
+    run(std::integral_constant<int, fwd_groups<HD>()>{});
   HOS_HIP_CHECK(hipGetLastError());
 }
 
@@ -767,16 +801,22 @@ void attn_bwd_hd(const float* qkv, long long ld, int kcol, int vcol, const float
   // dO is read from its f32 rows by both kernels (split to hi/lo as it is loaded); the dQ launch also forms
   // D = rowsum(dO∘O) for its queries and leaves it in dvec for the dK/dV launch
   dim3 grid(ceil_div(T, BR), nh, B);
-  constexpr int NGB = bwd_groups<HD>();
-  attn_dq_kernel<HD, NGB><<<grid, 256 * NGB, 0, st>>>(P.qh, P.ql, P.kh, P.kl, P.vh, P.vl, o, dout, ldo, lse, dvec,
-                                                            T, nh, nh / nkv, dqkv, ldd);
-  HOS_HIP_CHECK(hipGetLastError());
-  attn_dkdv_kernel<HD, NGB><<<grid, 256 * NGB, 0, st>>>(P.qh, P.ql, P.kh, P.kl, P.vh, P.vl, dout, ldo, lse,
-                                                              dvec, T, nh, nh / nkv, dqkv, ldd, kcol, vcol, part);
-  HOS_HIP_CHECK(hipGetLastError());
+  const auto run = [&](auto ng) {
+    constexpr int NG = decltype(ng)::value;
+    attn_dq_kernel<HD, NG><<<grid, 256 * NG, 0, st>>>(P.qh, P.ql, P.kh, P.kl, P.vh, P.vl, o, dout, ldo, lse, dvec, T, nh,
+                                                      nh / nkv, dqkv, ldd);
+    HOS_HIP_CHECK(hipGetLastError());
+    attn_dkdv_kernel<HD, NG><<<grid, 256 * NG, 0, st>>>(P.qh, P.ql, P.kh, P.kl, P.vh, P.vl, dout, ldo, lse, dvec, T, nh,
+                                                        nh / nkv, dqkv, ldd, kcol, vcol, part);
+    HOS_HIP_CHECK(hipGetLastError());
+  };
+  if (whole_axis<HD>(B, T, nh))
+    run(std::integral_constant<int, 1>{});
+  else
+    run(std::integral_constant<int, bwd_groups<HD>()>{});
   if (nh != nkv && !defer_group_sum) {
-    long long ne = (long long)B * T * nkv * 2 * HD;
-    attn_group_sum<HD><<<ceil_div(ne, 256), 256, 0, st>>>(part, B * T, nh, nkv, nh / nkv, dqkv, ldd, kcol, vcol);
+    long long ne = (long long)B * T * nkv * 2 * HD / 4;
+    attn_group_sum<HD><<<ceil_div(ne, 256), 256, 0, st>>>(reinterpret_cast<const float4*>(part), B * T, nh, nkv, nh / nkv, dqkv, ldd, kcol, vcol);
     HOS_HIP_CHECK(hipGetLastError());
   }
 }

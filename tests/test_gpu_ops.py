@@ -123,6 +123,14 @@ def test_attention_fwd_bwd(gpu, B, T, nh, nkv, hd):
         a.free()
 
 
+# launches of enough workgroups that none splits its streamed axis: at the rule's line and past it, of one token, of a
+# last block of one and two rows, and of more than 512 tokens
+@pytest.mark.parametrize("B,T,nh,nkv,hd", [(128, 33, 3, 1, 64), (128, 1, 6, 6, 64), (96, 130, 4, 2, 64),
+                                           (96, 129, 4, 2, 128), (11, 513, 14, 2, 64)])
+def test_attention_many_workgroups(gpu, B, T, nh, nkv, hd):
+    test_attention_fwd_bwd(gpu, B, T, nh, nkv, hd)
+
+
 @pytest.mark.parametrize("rows,V", [(17, 512), (4, 49152), (3, 151936)])
 def test_cross_entropy(gpu, rows, V):
     print(f"cross_entropy rows={rows} V={V}", flush=True)
