@@ -1045,6 +1045,32 @@ void launch_lora_cols_flush(ColsBatch& bt, hipStream_t st) {
   bt.used = 0;
 }
 
+namespace {
+// A factor pair out of an arena into host memory the device writes, in the caller's layout: A [in, r] from At [r][in], then
+// B [r, o] from rows of bpitch. Bound by the host link; 4 values a thread, 1 KB runs a wave.
+__global__ void factor_out_kernel(const float* __restrict__ At, int in, const float* __restrict__ B, long long bpitch, int o,
+                                  int r, long long na, long long n, float* __restrict__ out) {
+  const long long i0 = 4 * ((long long)blockIdx.x * blockDim.x + threadIdx.x);
+  float v[4];
+#pragma unroll
+  for (int e = 0; e < 4; e++) {
+    const long long i = i0 + e, b = i - na;
+    v[e] = i >= n ? 0.0f : i < na ? At[(i % r) * in + i / r] : B[(b / o) * bpitch + b % o];
+  }
+  if (i0 + 3 < n)
+    *reinterpret_cast<float4*>(out + i0) = make_float4(v[0], v[1], v[2], v[3]);
+  else
+    for (int e = 0; e < 4 && i0 + e < n; e++) out[i0 + e] = v[e];
+}
+}  // namespace
+
+void launch_factor_out(const float* At, int in, const float* B, long long bpitch, int o, int r, float* out, hipStream_t st) {
+  const long long na = At ? (long long)in * r : 0, n = na + (B ? (long long)o * r : 0);
+  if (n == 0) return;
+  factor_out_kernel<<<ceil_div(n, 1024), 256, 0, st>>>(At, in, B, bpitch, o, r, na, n, out);
+  HOS_HIP_CHECK(hipGetLastError());
+}
+
 void launch_lora_cols(long long M, int ns, float alpha, const float* Sm, long long lds, const float* Gm, long long ldg,
                       ColsSeg sg, float* C, long long scj, long long scc, float* ws, size_t ws_bytes,
                       hipStream_t st) {

@@ -142,4 +142,8 @@ void launch_lora_cols2(long long M, const ColsJob& a, const ColsJob* b, float* w
 size_t lora_rows_ws_bytes(long long M, long long K, int n);
 size_t lora_cols2_ws_bytes(long long M, const ColsJob& a, const ColsJob* b);
 
+// A factor pair (At [r][in], B's r rows of o columns, bpitch apart; either may be null) as A [in, r] and B [r, o], one after the
+// other, in host memory the device can write (16-byte aligned).
+void launch_factor_out(const float* At, int in, const float* B, long long bpitch, int o, int r, float* out, hipStream_t st);
+
 }  // namespace hos

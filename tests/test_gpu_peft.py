@@ -344,3 +344,25 @@ def test_llama32_1b_long_sequence_parity():
     """configs[3] architecture with LoRA r32 on all projections at T = 1024 (the benchmark's sequence length;
     M = 1024 rows, causal attention over the full sequence), B1."""
     _bench_shape_parity("llama3.2-1b", 1, 1024, seed=43)
+
+
+@pytest.mark.parametrize("rank", [1, 5, 16])
+def test_factors_read_back_as_set(gpu, rank):
+    """Odd and whole ranks, every target's widths, and the pairs in an order that needs the widest last: the bytes that went in."""
+    from hos_amd.peft import PeftModel
+    print(f"factor read-back rank {rank}", flush=True)
+    cfg = tiny(8, lora_rank=rank)
+    pm = PeftModel(gpu, cfg, max_batch=1, max_seq=32)
+    rng = np.random.default_rng(rank)
+    want = {}
+    for layer in range(cfg.n_layers):
+        for t in cfg.lora_targets:
+            i, ou = cfg.target_dims(t)
+            want[layer, t] = (rng.standard_normal((i, rank)).astype(np.float32),
+                              rng.standard_normal((rank, ou)).astype(np.float32))
+            pm.set_lora(layer, t, *want[layer, t])
+    for (layer, t), (A, B) in want.items():
+        a, b = pm.get_lora(layer, t)
+        np.testing.assert_array_equal(a, A)
+        np.testing.assert_array_equal(b, B)
+    pm.close()
